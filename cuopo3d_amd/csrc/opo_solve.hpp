@@ -226,23 +226,27 @@ template <typename T> struct SolveT final : SolveImpl {
             tw_fill(w3.s, [&](size_t i, double t, double r) { h[w3.o + i] = C{(T)t, (T)r}; });
         }
         // One x or y table at o_: entries exp(la + i phase(k)) / n, natural
-        // bins, forward sign -1; in dense form where the axis has roots.
-        DenseRoots rx, ry;
-        const DenseRoots *wx = nullptr, *wy = nullptr;
+        // bins, phase(n - k) = phase(k), forward sign -1; in dense form where
+        // the axis has roots.
+        using A = dense_acc<T>;
+        DenseRootsOf<A> rx, ry;
+        const DenseRootsOf<A> *wx = nullptr, *wy = nullptr;
         if (dense_x(g)) rx.fill(nx), wx = &rx;
         if (dense_y(g)) {
             if (ny != nx) ry.fill(ny);
             wy = ny == nx ? &rx : &ry;
         }
-        auto put_xy = [&](size_t o_, const LineShape &s, const DenseRoots *w8, double la, auto phase) {
+        auto put_xy = [&](size_t o_, const LineShape &s, const DenseRootsOf<A> *w8, double la, auto phase) {
             const int n = s.n();
             if (w8) {
                 unsigned *lo = reinterpret_cast<unsigned *>(h + o_ + 2 * (size_t)n);
-                const double am1 = std::expm1(la);
-                auto increment = [&](int k, double &re, double &im) {   // the entry times n, minus 1
-                    const double r = std::fmod(phase(k), kTwoPi), hs = std::sin(0.5 * r);
-                    re = am1 - (1.0 + am1) * 2.0 * hs * hs;
-                    im = (1.0 + am1) * std::sin(r);
+                const A am1 = std::expm1((A)la);
+                A er[kDenseMax], ei[kDenseMax];   // the entry times n, minus 1; even in the frequency
+                for (int k = 0; k <= n / 2; ++k) dense_increment<A>(phase(k), am1, er[k], ei[k]);
+                auto increment = [&](int k, A &re, A &im) {
+                    const int m = k <= n / 2 ? k : n - k;
+                    re = er[m];
+                    im = ei[m];
                 };
                 dense_fill<T>(n, -1, *w8, increment, [&](int i, T re, T im, unsigned l) {
                     h[o_ + i] = C{re, im};
