@@ -294,7 +294,7 @@ int opo_autotune(opo_solve *s, int reps, char *report, size_t report_len) {
     return rc;
 }
 int opo_tune_get(int precision, int axis, int n) {
-    return tune_get(precision == OPO_FP64, axis, n);
+    return tune_report(precision == OPO_FP64, axis, n);
 }
 int opo_tune_set(int precision, int axis, int n, int variant) {
     if (!tune_set(precision == OPO_FP64, axis, n, variant))

@@ -302,6 +302,14 @@ void tune_restore(bool fp64, int axis, int n, int stored) {
     if (std::atomic<int> *e = tune_entry(fp64, axis, n)) e->store(stored, std::memory_order_relaxed);
 }
 
+int tune_report(bool fp64, int axis, int n) {
+    const int v = tune_stored(fp64, axis, n), many = tune_get(fp64, axis, n);
+    if (v < 0 && axis == 0)
+        for (long long px : kPixelSteps)
+            if (time_default_variant(fp64, n, px) != many) return -1;
+    return many;
+}
+
 int tune_get(bool fp64, int axis, int n, long long pixels) {
     const int v = tune_stored(fp64, axis, n);
     if (v >= 0) return v;
@@ -309,7 +317,7 @@ int tune_get(bool fp64, int axis, int n, long long pixels) {
 }
 
 bool tune_set(bool fp64, int axis, int n, int v) {
-    if (!tune_variant_valid(fp64, axis, n, v)) return false;
+    if (!tune_variant_valid(fp64, axis, n, v < 0 ? 0 : v) || v < -1) return false;
     TuneTables &tt = tune_tables();
     if (axis == 0) tt.time[fp64][log2i(n)].store(v, std::memory_order_relaxed);
     else tt.xy[fp64][nx_index(n)].store(v, std::memory_order_relaxed);

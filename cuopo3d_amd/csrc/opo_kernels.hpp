@@ -105,12 +105,14 @@ hipError_t launch_power_pixel(hipStream_t st, const cplx<T> *f, size_t plane, in
 int tune_variant_count(int axis);
 bool tune_variant_valid(bool fp64, int axis, int n, int v);
 // The choice for an entry, tuned or the default (axis 0: for that many pixels,
-// 0: many).  tune_stored is -1 where nothing was
-// chosen; tune_restore puts such a value back.
+// 0: many).  tune_stored is -1 where nothing was chosen; tune_restore puts such
+// a value back, as tune_set does for -1.  tune_report is what the C ABI shows:
+// the choice or the default, and -1 where the default goes by the pixels.
 int tune_get(bool fp64, int axis, int n, long long pixels = 0);
 int tune_stored(bool fp64, int axis, int n);
 void tune_restore(bool fp64, int axis, int n, int stored);
 bool tune_set(bool fp64, int axis, int n, int v);
+int tune_report(bool fp64, int axis, int n);
 int tune_tile_px(bool fp64, int nt, int v);   // pixels per tile of a t-pass variant
 // The t-pass variant a launch over pixel rows of nx pixels uses: the tuned
 // choice for NT when its tile divides nx, else variant 0, whose tile (16,

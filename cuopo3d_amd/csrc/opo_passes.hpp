@@ -143,6 +143,8 @@ template <typename T, int NT, int V> struct TimeVariant {
 //  * FP64: 512 threads (64^2 x 256 55.9 / 58.8 on 256), 128 samples half the
 //    tile on 256 threads (96^2 69 / 73), 64 samples half the tile on 512
 //    below 256^2 (64^2 25.5 / 26.6, 512^2 1469 / 1283), 2048 one pixel on 384 (64^2 607 / 618).
+// A number of pixels from every range that the rule tells apart.
+constexpr long long kPixelSteps[] = {1, 1024, 4096, 16384, 65536};
 constexpr int time_default_variant(bool fp64, int nt, long long pixels) {
     if (nt < 64) return 0;
     const bool few = pixels > 0 && pixels < 4096, least = pixels > 0 && pixels < 1024;

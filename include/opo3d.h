@@ -257,7 +257,10 @@ int opo_profile_trips(opo_solve *s, int n, double ms[OPO_N_STAGES],
 #define OPO_TUNE_TIME_PASS 0
 #define OPO_TUNE_XY_PASS   1
 int opo_autotune(opo_solve *s, int reps, char *report, size_t report_len);
-/* Current variant for (precision, axis, size n = NT or NX); set returns
+/* Current variant for (precision, axis, size n = NT or NX).  -1: none was
+ * chosen for a t pass whose default goes by the pixels of the work (a small
+ * grid takes another launch shape than a large one); setting -1 returns to
+ * that state, so a value from get can always be set again.  set returns
  * OPO_ERR_ARG for a variant that does not exist. */
 int opo_tune_get(int precision, int axis, int n);
 int opo_tune_set(int precision, int axis, int n, int variant);
