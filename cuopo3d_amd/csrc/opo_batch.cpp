@@ -593,7 +593,8 @@ struct opo_batch {
         for (int axis = 0; axis < 2 && !rc; ++axis) {
             for (int n : axis == 0 ? nts : nxs) {
                 const int stage = axis == 0 ? OPO_STAGE_TIME_OP : OPO_STAGE_XY_OP;
-                int best = axis == 0 ? class_time_variant(n) : tune_get(fp64, 1, n);
+                const int before = tune_stored(fp64, axis, n);
+                int best = -1;
                 double best_us = 1e30;
                 report += axis == 0 ? "batch t pass NT=" : "batch xy pass NX=";
                 report += std::to_string(n) + " (us per launch):";
@@ -617,9 +618,10 @@ struct opo_batch {
                         best = v;
                     }
                 }
-                tune_set(fp64, axis, n, best);
-                report += " -> v" + std::to_string(best) + "\n";
+                if (rc || best < 0) tune_restore(fp64, axis, n, before);   // the previous choice stands
+                else tune_set(fp64, axis, n, best);
                 if (rc) break;
+                report += best < 0 ? " none to time\n" : " -> v" + std::to_string(best) + "\n";
             }
         }
         off = 0;

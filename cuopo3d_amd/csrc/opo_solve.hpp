@@ -806,7 +806,8 @@ template <typename T> struct SolveT final : SolveImpl {
             const int axis = order[round];
             if (axis == 1 && g.nx != g.ny) continue;   // NX != NY planes have one launch shape
             const int n = axis == 0 ? g.nt : g.nx;
-            int best = tune_get(fp64, axis, n, (long long)P);
+            const int before = tune_stored(fp64, axis, n);
+            int best = -1;
             double best_t = 1e30;
             report += axis == 0 ? "t pass NT=" : "xy pass NX=";
             report += std::to_string(n) + " (us per slice):";
@@ -830,6 +831,12 @@ template <typename T> struct SolveT final : SolveImpl {
                     best_t = us;
                     best = v;
                 }
+            }
+            // one pixel has no t-pass candidates: nothing is chosen
+            if (best < 0) {
+                tune_restore(fp64, axis, n, before);
+                report += " none to time\n";
+                continue;
             }
             tune_set(fp64, axis, n, best);
             report += " -> v" + std::to_string(best) + "\n";
