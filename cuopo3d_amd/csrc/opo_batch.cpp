@@ -678,12 +678,12 @@ size_t opo_batch_footprint(const opo_grid *g, int precision, int n_trips) {
     const size_t cb = precision == OPO_FP64 ? 16 : 8;
     // Every device allocation of a resident solve, each rounded up to the
     // allocation granularity assumed here: Api, Ap, As, Ai; the table block
-    // (twiddles, D, GDD, Q, free-space and modulator tables as hi/lo pairs);
+    // (rotations, D, GDD, Q, free-space and modulator tables);
     // the power partials (one per 4096 cells, 1 to 1024, three fields) and
     // counters; the per-trip power series of the batch.
     const size_t kGran = 64 * 1024;
     auto up = [&](size_t b) { return (b + kGran - 1) / kGran * kGran; };
-    const size_t tabs = 2 * (size_t)(6 * g->nx + 5 * g->ny + 6 * g->nt) * cb;
+    const size_t tabs = (precision == OPO_FP64 ? SolveT<double>::table_entries(*g) : SolveT<float>::table_entries(*g)) * cb;
     size_t nblk = (n + 4095) / 4096;
     nblk = nblk < 1 ? 1 : (nblk > 1024 ? 1024 : nblk);
     const size_t dbuf = sizeof(double) * (3 * nblk + 4);
