@@ -502,17 +502,18 @@ __global__ void __launch_bounds__(64 * kDenseBandWaves) k_xyband(FieldOps<T> ops
 }
 
 // Lines that do not fit a wave's registers (FP64 256 points, 512 points in
-// either precision) run in LDS: Q_x on bands of RB consecutive rows, then Q_y
-// on bands of CB consecutive columns (rows of the band are CB elements
-// contiguous in HBM).
+// either precision), and few lines (dense_axis), run in LDS: Q_x on bands of RB
+// consecutive rows, then Q_y on bands of CB consecutive columns (rows of the
+// band are CB elements contiguous in HBM).
 template <typename T, int NX, int RB, int BS>
 __global__ void __launch_bounds__(BS) k_xrows(FieldOps<T> ops, int ny, const cplx<T> *__restrict__ tw,
                                               const int *status) {
     const int stop = stop_flag(status);
     constexpr int NXP = NX + 1;
     __shared__ cplx<T> lds[RB * NXP];
-    __shared__ cplx<T> twl[tw_elems<T, NX, USE_BAND>() + 1];
-    stage_rotations<T, NX>(tw, twl, threadIdx.x, BS);
+    constexpr bool STW = band_rotations_in_lds<T, NX>();
+    __shared__ cplx<T> twl[STW ? tw_elems<T, NX, USE_BAND>() : 1];
+    if constexpr (STW) stage_rotations<T, NX>(tw, twl, threadIdx.x, BS);
     const int bands = ny / RB;
     const int t = blockIdx.x / bands, r0 = (blockIdx.x % bands) * RB, f = blockIdx.y;
     cplx<T> *A = ops.f[f] + ((size_t)t * ny + r0) * NX;
@@ -520,7 +521,7 @@ __global__ void __launch_bounds__(BS) k_xrows(FieldOps<T> ops, int ny, const cpl
                                  [&](int i, cplx<T> v) { lds[(i / NX) * NXP + (i % NX)] = v; });
     __syncthreads();
     if (stop) return;
-    band_line_op<T, NX, -1, NXP, 1, TwShear>(lds, RB, twl, ops.tab[f], threadIdx.x, BS);
+    band_line_op<T, NX, -1, NXP, 1, TwShear>(lds, RB, STW ? twl : tw, ops.tab[f], threadIdx.x, BS);
     chunked_copy<T, RB * NX, BS>(threadIdx.x, [&](int i) { return lds[(i / NX) * NXP + (i % NX)]; },
                                  [&](int i, cplx<T> v) { A[i] = v; });
 }
@@ -531,8 +532,9 @@ __global__ void __launch_bounds__(BS) k_ycols(FieldOps<T> ops, int nx, const cpl
     const int stop = stop_flag(status);
     constexpr int CBP = CB + 1;
     __shared__ cplx<T> lds[NY * CBP];
-    __shared__ cplx<T> twl[tw_elems<T, NY, USE_BAND>() + 1];
-    stage_rotations<T, NY>(tw, twl, threadIdx.x, BS);
+    constexpr bool STW = band_rotations_in_lds<T, NY>();
+    __shared__ cplx<T> twl[STW ? tw_elems<T, NY, USE_BAND>() : 1];
+    if constexpr (STW) stage_rotations<T, NY>(tw, twl, threadIdx.x, BS);
     const int bands = nx / CB;
     const int t = blockIdx.x / bands, c0 = (blockIdx.x % bands) * CB, f = blockIdx.y;
     cplx<T> *A = ops.f[f] + (size_t)t * NY * nx + c0;
@@ -541,7 +543,7 @@ __global__ void __launch_bounds__(BS) k_ycols(FieldOps<T> ops, int nx, const cpl
     __syncthreads();
     if (stop) return;
     // lines are the CB columns (line c starts at c, its elements CBP apart)
-    band_line_op<T, NY, -1, 1, CBP, TwShear>(lds, CB, twl, ops.taby[f], threadIdx.x, BS);
+    band_line_op<T, NY, -1, 1, CBP, TwShear>(lds, CB, STW ? twl : tw, ops.taby[f], threadIdx.x, BS);
     chunked_copy<T, NY * CB, BS>(threadIdx.x, [&](int i) { return lds[(i / CB) * CBP + (i % CB)]; },
                                  [&](int i, cplx<T> v) { A[(size_t)(i / CB) * nx + (i % CB)] = v; });
 }
@@ -667,12 +669,12 @@ bool xyplane_supported(int nx, int ny, bool fp64) {
     return nx == 1 || line_len_supported(nx);
 }
 
-// Planes with an axis beyond 128 points: Q_x on bands of rows, then Q_y on
-// bands of columns.  Lines that fit a wave's registers take 16 per wave
-// (k_xyband; FP32 256 x 256 x 64, rows + cols: 100 us in LDS, 73 here), the
-// others bands in LDS (k_xrows, k_ycols) of 32 rows or columns where the
-// other dimension allows, else 16 (every supported length is a multiple of 16).
-// 256- and 512-point lines there:
+// Planes with an axis beyond 128 points, and planes of few lines (dense_axis):
+// Q_x on bands of rows, then Q_y on bands of columns.  Lines that fit a wave's
+// registers take 16 per wave (k_xyband; FP32 256 x 256 x 64, rows + cols: 100 us
+// in LDS, 73 here), the others bands in LDS (k_xrows, k_ycols) of 32 rows or
+// columns where the other dimension allows, else 16 (every supported length is a
+// multiple of 16).  256- and 512-point lines there:
 // FP32 bands of 32 on 512 threads (256: one 16-point DFT per thread and
 // phase; 512: 131 KiB of LDS, as fast as bands of 16 on 256 threads), FP64
 // bands of 16 (256: 64 KiB of LDS, two workgroups per CU; 512: 131 KiB).
@@ -685,9 +687,9 @@ template <typename T, int NX>
 static hipError_t rows_launch(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                               const cplx<T> *tw, const int *status) {
     if constexpr (dense_line<T>(NX)) {
-        if (dense_axis<T>(NX, g.ny, g.nt)) return xy_band_launch<T, NX, true>(st, g, ops, nf, status);
+        if (dense_axis<T>(NX, g.ny, g.nt, true)) return xy_band_launch<T, NX, true>(st, g, ops, nf, status);
     }
-    if constexpr ((!dense_line<T>(NX) || NX == 256) && max_band<T, NX>() == 32) {
+    if constexpr (band_line<T>(NX) && max_band<T, NX>() == 32) {
         constexpr int B32 = band32_threads<T, NX>();
         if (g.ny % 32 == 0) {
             hipLaunchKernelGGL((k_xrows<T, NX, 32, B32>), dim3((unsigned)(g.nt * (g.ny / 32)), (unsigned)nf),
@@ -695,7 +697,7 @@ static hipError_t rows_launch(hipStream_t st, const Geometry &g, const FieldOps<
             return hipGetLastError();
         }
     }
-    if constexpr (!dense_line<T>(NX) || NX == 256) {
+    if constexpr (band_line<T>(NX) && !(sizeof(T) == 8 && dense_line<T>(NX))) {   // those only beside 64 or more
         hipLaunchKernelGGL((k_xrows<T, NX, 16, 256>), dim3((unsigned)(g.nt * (g.ny / 16)), (unsigned)nf), dim3(256),
                            0, st, ops, g.ny, tw, status);
         return hipGetLastError();
@@ -706,9 +708,9 @@ template <typename T, int NY>
 static hipError_t cols_launch(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                               const cplx<T> *tw, const int *status) {
     if constexpr (dense_line<T>(NY)) {
-        if (dense_axis<T>(NY, g.nx, g.nt)) return xy_band_launch<T, NY, false>(st, g, ops, nf, status);
+        if (dense_axis<T>(NY, g.nx, g.nt, false)) return xy_band_launch<T, NY, false>(st, g, ops, nf, status);
     }
-    if constexpr ((!dense_line<T>(NY) || NY == 256) && max_band<T, NY>() == 32) {
+    if constexpr (band_line<T>(NY) && max_band<T, NY>() == 32) {
         constexpr int B32 = band32_threads<T, NY>();
         if (g.nx % 32 == 0) {
             hipLaunchKernelGGL((k_ycols<T, NY, 32, B32>), dim3((unsigned)(g.nt * (g.nx / 32)), (unsigned)nf),
@@ -716,19 +718,23 @@ static hipError_t cols_launch(hipStream_t st, const Geometry &g, const FieldOps<
             return hipGetLastError();
         }
     }
-    if constexpr (!dense_line<T>(NY) || NY == 256) {
+    if constexpr (band_line<T>(NY) && !(sizeof(T) == 8 && dense_line<T>(NY))) {   // those only beside 64 or more
         hipLaunchKernelGGL((k_ycols<T, NY, 16, 256>), dim3((unsigned)(g.nt * (g.nx / 16)), (unsigned)nf), dim3(256),
                            0, st, ops, g.nx, tw, status);
         return hipGetLastError();
     }
     return hipErrorInvalidValue;   // not reached: every other line is dense
 }
+// Planes whose lines both run on the matrix cores, in one launch.
+template <typename T> static bool dense_plane_grid(const Geometry &g) {
+    return g.nx <= 128 && g.ny <= 128 && dense_axis<T>(g.nx, g.ny, g.nt, true) && dense_axis<T>(g.ny, g.nx, g.nt, false);
+}
 template <typename T>
 static hipError_t xy_rect_launch(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                                  const cplx<T> *tw_x, const cplx<T> *tw_y, const int *status) {
     if (!line_len_supported(g.nx) || !line_len_supported(g.ny) || g.nx % 16 || g.ny % 16)
         return hipErrorInvalidValue;
-    if (g.nx != g.ny && g.nx <= 128 && g.ny <= 128) {
+    if (g.nx != g.ny && dense_plane_grid<T>(g)) {
         switch (g.nx) {
             case 16: return xy_dense_rect_y<T, 16>(st, g, ops, nf, status);
             case 32: return xy_dense_rect_y<T, 32>(st, g, ops, nf, status);
@@ -763,7 +769,7 @@ static hipError_t xy_rect_launch(hipStream_t st, const Geometry &g, const FieldO
 template <typename T>
 hipError_t launch_xyplane(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                           const cplx<T> *tw, const cplx<T> *tw_y, const int *status) {
-    if (g.nx != g.ny) return xy_rect_launch<T>(st, g, ops, nf, tw, tw_y, status);
+    if (g.nx != g.ny || (g.nx == 128 && !dense_plane_grid<T>(g))) return xy_rect_launch<T>(st, g, ops, nf, tw, tw_y, status);
     switch (g.nx) {
         case 1: return xy_pixel_launch<T>(st, g, ops, nf, status);
         case 16: return xy_dense_launch<T, 16>(st, g, ops, nf, status);

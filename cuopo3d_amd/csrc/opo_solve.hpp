@@ -170,8 +170,8 @@ template <typename T> struct SolveT final : SolveImpl {
     // diagonal tables in slot order (tw_slot_bin), each entry a (hi, lo) pair.
     // x and y lines on the matrix cores have dense tables (opo_mfma.hpp) and
     // no rotations.
-    static bool dense_x(const opo_grid &g) { return dense_axis<T>(g.nx, g.ny, g.nt); }
-    static bool dense_y(const opo_grid &g) { return dense_axis<T>(g.ny, g.nx, g.nt); }
+    static bool dense_x(const opo_grid &g) { return dense_axis<T>(g.nx, g.ny, g.nt, true); }
+    static bool dense_y(const opo_grid &g) { return dense_axis<T>(g.ny, g.nx, g.nt, false); }
     static size_t table_entries(const opo_grid &g) { return table_offsets(g).end; }
     struct TableOffsets {
         size_t twx, twy, twt, D, G, qx, qy, fx, fy, E, end;
