@@ -599,7 +599,7 @@ struct opo_batch {
                 report += axis == 0 ? "batch t pass NT=" : "batch xy pass NX=";
                 report += std::to_string(n) + " (us per launch):";
                 for (int v = 0; v < tune_variant_count(axis) && !rc; ++v) {
-                    if (!tune_variant_valid(fp64, axis, n, v)) continue;
+                    if (!tune_variant_timed(fp64, axis, n, v)) continue;
                     bool fits = true;
                     if (axis == 0)
                         for (const BatchEntry *e : resident)

@@ -121,42 +121,6 @@ __global__ void __launch_bounds__(BS) kb_timep(const SolveDesc<T> *__restrict__ 
     nl_time_run<T, NT, TX, BS>(TimeBatch<T, NT, TX>{sd, status, work, n_work, mode}, lds, stab);
 }
 
-// Work units of the xy pass over a work list: item = k nt + t, plane t of
-// field k (or of s and i with the free-space tables).
-template <typename T, int NX> struct XyBatch {
-    const SolveDesc<T> *sd;
-    const TripState *ts;
-    const int *status;
-    const WorkItem *work;
-    int n, free_space;
-    __device__ int units() const { return n; }
-    __device__ bool skip(int u) const {
-        const int s = work[u].solve;
-        return status[s] != 0 || (free_space && !ts[s].fs);
-    }
-    __device__ cplx<T> *plane(int u) const {
-        const SolveDesc<T> &d = sd[work[u].solve];
-        const int k = work[u].item / d.nt, t = work[u].item % d.nt;
-        const int f = free_space ? 1 + k : k;
-        return (f == 0 ? d.f[0] : (f == 1 ? d.f[1] : d.f[2])) + (size_t)t * NX * NX;
-    }
-    __device__ void tables(int u, const cplx<T> *&tx, const cplx<T> *&ty) const {
-        const SolveDesc<T> &d = sd[work[u].solve];
-        const int k = work[u].item / d.nt;
-        tx = (free_space ? d.qfsx : d.qx) + xy_table_elems<T>(NX) * k;
-        ty = (free_space ? d.qfsy : d.qy) + xy_table_elems<T>(NX) * k;
-    }
-};
-
-template <typename T, int NX>
-__global__ void __launch_bounds__((dense_threads<NX, NX>()), (dense_waves<T, NX>()))
-    kb_xydensep(const SolveDesc<T> *__restrict__ sd, const TripState *__restrict__ ts,
-                const int *__restrict__ status, const WorkItem *__restrict__ work, int n_work, int free_space) {
-    __shared__ DensePlane<T, NX> S;
-    __shared__ DenseTabs<T, NX> Tb;
-    dense_run<T, NX>(XyBatch<T, NX>{sd, ts, status, work, n_work, free_space}, S, Tb, threadIdx.x, 0);
-}
-
 // Plane group t of field k (or of s and i with the free-space tables).
 template <typename T, int NX, int PC, int P>
 __global__ void __launch_bounds__((PC * dense_threads<NX, NX>()), (dense_waves<T, NX>()))
@@ -390,18 +354,10 @@ template <typename T, int NX>
 static hipError_t bx_dispatch(hipStream_t st, int n_work, const SolveDesc<T> *sd, const TripState *ts,
                               const int *status, const WorkItem *work, int fs, int v) {
     if (!tune_variant_valid(sizeof(T) == 8, 1, NX, v)) return hipErrorInvalidValue;
-    const int bs = xy_variant_bs(NX, v);
     const dim3 g((unsigned)n_work);
-    if constexpr (NX >= 64) {
-        if constexpr (sizeof(T) == 4) {
-            if (xy_variant_persistent(NX, v)) {
-                hipLaunchKernelGGL((kb_xydensep<T, NX>), dim3(persistent_grid(n_work, xy_variant_per_cu(NX, v))),
-                                   dim3(4 * NX), 0, st, sd, ts, status, work, n_work, fs);
-                return hipGetLastError();
-            }
-        }
-    } else {
+    if constexpr (NX <= 32) {
         constexpr int P = xy_group(NX, 3), PC = 256 / (4 * NX);
+        const int bs = xy_variant_bs(sizeof(T) == 8, NX, v);
         if (xy_group(NX, v) > 1) {
             if (bs == 256) hipLaunchKernelGGL((kb_xydense<T, NX, PC, P>), g, dim3(256), 0, st, sd, ts, status, work, fs);
             else if (bs == 512) hipLaunchKernelGGL((kb_xydense<T, NX, 2 * PC, P>), g, dim3(512), 0, st, sd, ts, status, work, fs);

@@ -196,8 +196,6 @@ unsigned persistent_grid(int units, int per_cu) {
 }
 
 // ----------------------------------------------------- variant tables
-constexpr int kSplitVariants = 3;   // xy variants of the two-pass form (xy_split_launch)
-
 // Chosen variant per (precision, size): process-wide, read at every launch
 // and written by the tuner, so the entries are atomics (a launch sees either
 // the old or the new choice, both of which give the same results).
@@ -274,13 +272,11 @@ bool tune_variant_valid(bool fp64, int axis, int n, int v) {
         int tx = 0, bs = 0;
         return fp64 ? time_info<double>(n, v, tx, bs) : time_info<float>(n, v, tx, bs);
     }
-    if (v < 0 || v >= kXyVariants || nx_index(n) < 0) return false;
-    if (n < 16 || n == 512) return v == 0;   // 512: the two-pass form, one band shape
-    // FP32 256 and FP64 128 have one launch shape under all of these numbers.
-    if (n == 256 || (fp64 && n == 128)) return v < kSplitVariants;
-    if (n <= 32) return v < 6;
-    if (xy_variant_persistent(n, v)) return !fp64 && n * n / xy_variant_bs(n, v) <= 16;
-    return true;
+    return nx_index(n) >= 0 && xy_variant_numbered(fp64, n, v);
+}
+
+bool tune_variant_timed(bool fp64, int axis, int n, int v) {
+    return tune_variant_valid(fp64, axis, n, v) && (axis == 0 || xy_variant_shape(fp64, n, v) == v);
 }
 
 static std::atomic<int> *tune_entry(bool fp64, int axis, int n) {
@@ -337,14 +333,14 @@ int time_variant_for(bool fp64, int nt, int nx, long long pixels) {
 }
 
 int tune_per_cu(bool fp64, int axis, int n, int v) {
-    if (axis == 1) return xy_variant_per_cu(n, v);
+    if (axis == 1) return 0;
     int tx = 0, bs = 0, per_cu = 0;
     const bool ok = fp64 ? time_info<double>(n, v, tx, bs, per_cu) : time_info<float>(n, v, tx, bs, per_cu);
     return ok ? per_cu : 0;
 }
 
 int tune_block(bool fp64, int axis, int n, int v) {
-    if (axis == 1) return (n == 256 || (fp64 && n == 128)) ? (v == 1 ? 512 : 256) : xy_variant_bs(n, v);
+    if (axis == 1) return xy_variant_bs(fp64, n, v);
     int tx = 0, bs = 0;
     const bool ok = fp64 ? time_info<double>(n, v, tx, bs) : time_info<float>(n, v, tx, bs);
     return ok ? bs : 0;
@@ -468,7 +464,7 @@ __global__ void __launch_bounds__(256) k_xypixel(FieldOps<T> ops, int nt, const 
 }
 
 // Planes of 16 to 128 points (opo_mfma.hpp): P consecutive planes by PC sets
-// of waves, or a run of planes per workgroup.
+// of waves.
 template <typename T, int NX, int NY, int PC, int P>
 __global__ void __launch_bounds__((PC * dense_threads<NX, NY>()), (dense_waves<T, (NX > NY ? NX : NY)>()))
     k_xydense(FieldOps<T> ops, const int *status) {
@@ -478,14 +474,6 @@ __global__ void __launch_bounds__((PC * dense_threads<NX, NY>()), (dense_waves<T
     const int f = blockIdx.y;
     dense_group<T, NX, NY, PC, P>(ops.f[f] + (size_t)blockIdx.x * P * NX * NY, ops.tab[f], ops.taby[f], S, Tb,
                                   threadIdx.x, stop);
-}
-template <typename T, int NX>
-__global__ void __launch_bounds__((dense_threads<NX, NX>()), (dense_waves<T, NX>()))
-    k_xydensep(FieldOps<T> ops, int nt, int nf, const int *status) {
-    const int stop = stop_flag(status);
-    __shared__ DensePlane<T, NX> S;
-    __shared__ DenseTabs<T, NX> Tb;
-    dense_run<T, NX>(XySolo<T, NX>{ops, nt, nf}, S, Tb, threadIdx.x, stop);
 }
 // Lines of planes beyond that, a band of 16 rows or columns per wave.
 template <typename T, int N, bool ROWS>
@@ -563,7 +551,7 @@ static hipError_t xy_split_launch_b(hipStream_t st, const Geometry &g, const Fie
     return hipGetLastError();
 }
 // Variants of the FP64 256 x 256 planes: v = 0 bands of 32 with 256 threads,
-// 1 bands of 32 with 512, 2 bands of 16 with 256; kSplitVariants of them.
+// 1 bands of 32 with 512, 2 bands of 16 with 256.
 template <typename T, int NX>
 static hipError_t xy_split_launch(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                                   const cplx<T> *tw, const int *status, int v = 0) {
@@ -584,13 +572,11 @@ static hipError_t xy_band_launch(hipStream_t st, const Geometry &g, const FieldO
 }
 
 // The launch shapes of square planes on the matrix cores, 4 NX threads per
-// plane (a wave per 16 lines): NX >= 64 one plane
-// per workgroup or (FP32, v >= 3) persistent workgroups, NX <= 32 one plane
-// (v < 3) or groups of 256 / NX planes on 256, 512 or 1024 threads.
+// plane (a wave per 16 lines): one plane per workgroup, or for NX <= 32 (v >= 3)
+// groups of 256 / NX planes on 256, 512 or 1024 threads.
 template <typename T, int NX>
 static hipError_t xy_dense_launch(hipStream_t st, const Geometry &g, const FieldOps<T> &ops, int nf,
                                   const int *status) {
-    const int v = tune_get(sizeof(T) == 8, 1, NX);
     // Few FP64 128-point planes, one workgroup of a CU each, leave CUs idle:
     // the same lines as bands of four waves (128 x 128 x 16: 43.7 -> 42.3 us per
     // slice).
@@ -600,20 +586,13 @@ static hipError_t xy_dense_launch(hipStream_t st, const Geometry &g, const Field
             return e != hipSuccess ? e : xy_band_launch<T, NX, false>(st, g, ops, nf, status);
         }
     }
-    if constexpr (NX >= 64) {
-        if constexpr (sizeof(T) == 4) {
-            if (xy_variant_persistent(NX, v)) {
-                hipLaunchKernelGGL((k_xydensep<T, NX>), dim3(persistent_grid(g.nt * nf, xy_variant_per_cu(NX, v))),
-                                   dim3(4 * NX), 0, st, ops, g.nt, nf, status);
-                return hipGetLastError();
-            }
-        }
-    } else {
+    if constexpr (NX <= 32) {
         constexpr int P = xy_group(NX, 3), PC = 256 / (4 * NX);   // planes at once on 256 threads
+        const int v = tune_get(sizeof(T) == 8, 1, NX);
         if (xy_group(NX, v) > 1) {
             if (g.nt % P != 0) return hipErrorInvalidValue;
             const dim3 grid((unsigned)(g.nt / P), (unsigned)nf);
-            const int bs = xy_variant_bs(NX, v);
+            const int bs = xy_variant_bs(sizeof(T) == 8, NX, v);
             if (bs == 256) hipLaunchKernelGGL((k_xydense<T, NX, NX, PC, P>), grid, dim3(256), 0, st, ops, status);
             else if (bs == 512) hipLaunchKernelGGL((k_xydense<T, NX, NX, 2 * PC, P>), grid, dim3(512), 0, st, ops, status);
             else hipLaunchKernelGGL((k_xydense<T, NX, NX, 4 * PC, P>), grid, dim3(1024), 0, st, ops, status);

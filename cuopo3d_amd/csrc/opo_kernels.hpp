@@ -104,6 +104,8 @@ hipError_t launch_power_pixel(hipStream_t st, const cplx<T> *f, size_t plane, in
 // axis 0: fused t pass, keyed by NT; axis 1: xy pass, keyed by NX.
 int tune_variant_count(int axis);
 bool tune_variant_valid(bool fp64, int axis, int n, int v);
+// Whether v stands for a launch shape that no smaller number stands for.
+bool tune_variant_timed(bool fp64, int axis, int n, int v);
 // The choice for an entry, tuned or the default (axis 0: for that many pixels,
 // 0: many).  tune_stored is -1 where nothing was chosen; tune_restore puts such
 // a value back, as tune_set does for -1.  tune_report is what the C ABI shows:

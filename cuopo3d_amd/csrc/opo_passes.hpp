@@ -160,20 +160,34 @@ constexpr int time_default_variant(bool fp64, int nt, long long pixels) {
     return few ? 4 : 1;
 }
 
-// Variants of the xy pass: V < 3 one plane per workgroup (FP64 256-point
-// planes: the band shapes of xy_split_launch); for NX >= 64 in FP32, V >= 3
-// persistent workgroups (k + 1 per CU, k = (V - 3) % 2) walking a run of
-// planes; for 16 <= NX <= 32, V = 3 + b groups of 256 / NX planes per
-// workgroup (xy_group) on 256, 512 or 1024 threads.  Planes of up to 128
-// points run on as many waves as their lines need (opo_mfma.hpp), whatever
-// the variant's block size says.
+// Variants of the xy pass.  16 <= NX <= 32: V < 3 one plane per workgroup, V = 3
+// + b groups of 256 / NX planes (xy_group) on 256, 512 or 1024 threads.  FP64 256:
+// the band shapes of xy_split_launch.  The other sizes have one launch shape,
+// and every number that stood for a block size or for persistent workgroups of
+// lines in LDS is taken for it (saved choices stay valid): xy_variant_shape is the
+// number that the tuner times for V.  (Persistent workgroups walking a run of
+// matrix-core planes, one or two per CU, are slower: batched 64-point planes 311
+// and 221 against 201 us per launch, 96 566 and 456 against 442, 128 675 and 610
+// against 552.)
 constexpr int kXyVariants = 9;
-constexpr bool xy_variant_persistent(int nx, int v) { return nx >= 64 && v >= 3; }
-constexpr int xy_variant_bs(int nx, int v) {
-    const int b = xy_variant_persistent(nx, v) ? (v - 3) / 2 : v % 3;
-    return b == 0 ? 256 : (b == 1 ? 512 : 1024);
+constexpr bool xy_variant_numbered(bool fp64, int nx, int v) {
+    if (v < 0 || v >= kXyVariants) return false;
+    if (nx < 16 || nx == 512) return v == 0;
+    if (nx == 256 || (fp64 && nx == 128)) return v < 3;
+    if (nx <= 32) return v < 6;
+    return v < 3 || (!fp64 && nx * nx / (256 << ((v - 3) / 2)) <= 16);
 }
-constexpr int xy_variant_per_cu(int nx, int v) { return xy_variant_persistent(nx, v) ? (v - 3) % 2 + 1 : 0; }
+constexpr int xy_variant_shape(bool fp64, int nx, int v) {
+    if (fp64 && nx == 256) return v;
+    return nx <= 32 && v >= 3 ? v : 0;
+}
+// Threads per workgroup.
+constexpr int xy_variant_bs(bool fp64, int nx, int v) {
+    if (nx == 256) return fp64 && v == 1 ? 512 : 256;
+    if (nx == 512) return fp64 ? 256 : 512;
+    if (nx < 16) return 256;
+    return nx <= 32 && v >= 3 ? 256 << (v - 3) : 4 * nx;
+}
 // Untuned choice: one plane per workgroup; FP64 256-point planes in bands of
 // 16 (256 x 256 x 64 242 us per slice).
 constexpr int xy_default_variant(bool fp64, int nx) { return fp64 && nx == 256 ? 2 : 0; }
@@ -608,25 +622,6 @@ template <typename T, int NT, int TX> struct TimeSolo {
     __device__ int tile(int u) const { return u; }
     __device__ void stage(int, cplx<T> *stab, int tid, int nthr) const {
         stage_time_tables<T, NT, TX>(tw, a, stab, tid, nthr);
-    }
-};
-
-// Work units of the xy pass of one solve: plane t of field f, u = f nt + t;
-// plane(u) is the plane's first element, tables(u, tx, ty) its tables.
-template <typename T, int NX> struct XySolo {
-    const FieldOps<T> &ops;
-    int nt, nf;
-    __device__ int units() const { return nt * nf; }
-    __device__ bool skip(int) const { return false; }
-    __device__ cplx<T> *plane(int u) const {
-        const int f = u / nt;
-        cplx<T> *base = f == 0 ? ops.f[0] : (f == 1 ? ops.f[1] : ops.f[2]);
-        return base + (size_t)(u % nt) * NX * NX;
-    }
-    __device__ void tables(int u, const cplx<T> *&tx, const cplx<T> *&ty) const {
-        const int f = u / nt;
-        tx = f == 0 ? ops.tab[0] : (f == 1 ? ops.tab[1] : ops.tab[2]);
-        ty = f == 0 ? ops.taby[0] : (f == 1 ? ops.taby[1] : ops.taby[2]);
     }
 };
 

@@ -812,7 +812,7 @@ template <typename T> struct SolveT final : SolveImpl {
             report += axis == 0 ? "t pass NT=" : "xy pass NX=";
             report += std::to_string(n) + " (us per slice):";
             for (int v = 0; v < tune_variant_count(axis); ++v) {
-                if (!tune_variant_valid(fp64, axis, n, v)) continue;
+                if (!tune_variant_timed(fp64, axis, n, v)) continue;
                 if (axis == 0 && (g.nx == 1 || g.nx % tune_tile_px(fp64, n, v) != 0)) continue;
                 tune_set(fp64, axis, n, v);
                 float ms = 1e30f;

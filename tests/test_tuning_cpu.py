@@ -55,3 +55,16 @@ def test_no_entry_for_other_sizes():
         assert lib.opo_tune_set(OPO_FP32, axis, n, 0) == capi.OPO_ERR_ARG
     assert lib.opo_tune_set(OPO_FP64, OPO_TUNE_TIME_PASS, 4096, -1) == capi.OPO_ERR_ARG   # FP32 only
     assert lib.opo_tune_set(OPO_FP32, OPO_TUNE_TIME_PASS, 256, -2) == capi.OPO_ERR_ARG
+
+
+@pytest.mark.parametrize("prec,nx,accepted", [
+    (OPO_FP32, 1, [0]), (OPO_FP32, 16, range(6)), (OPO_FP32, 32, range(6)), (OPO_FP32, 64, range(9)),
+    (OPO_FP32, 96, [0, 1, 2, 7, 8]), (OPO_FP32, 128, [0, 1, 2, 7, 8]), (OPO_FP32, 256, range(3)), (OPO_FP32, 512, [0]),
+    (OPO_FP64, 32, range(6)), (OPO_FP64, 64, range(3)), (OPO_FP64, 96, range(3)), (OPO_FP64, 128, range(3)),
+    (OPO_FP64, 256, range(3)), (OPO_FP64, 512, [0])])
+def test_xy_numbers_of_saved_choices_stay_valid(prec, nx, accepted):
+    lib = capi.load()
+    saved = lib.opo_tune_get(prec, OPO_TUNE_XY_PASS, nx)
+    got = [v for v in range(-2, 64) if v != -1 and lib.opo_tune_set(prec, OPO_TUNE_XY_PASS, nx, v) == capi.OPO_OK]
+    assert lib.opo_tune_set(prec, OPO_TUNE_XY_PASS, nx, saved) == capi.OPO_OK
+    assert got == list(accepted)
