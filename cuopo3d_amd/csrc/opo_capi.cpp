@@ -93,10 +93,12 @@ int make_solve(const opo_grid *g, const opo_params *p, int device,
 // Each device holds its own copy of the array at its own address, found
 // once per device with hipGetSymbolAddress; host code never uses the
 // array's name as an address.
-// The array holds OPO_NOALLOC_SCRATCH_BYTES of what noalloc_bytes counts and
-// kDenseExtra for the dense x and y tables, which take up to 8 (nx + ny) bytes
-// FP32 elements more than the (hi, lo) tables the count is based on.
+// The array holds OPO_NOALLOC_SCRATCH_BYTES of what noalloc_bytes counts, 12
+// elements per axis point, and kDenseExtra for FP32 x and y lines of a matrix-core
+// size, whose tables take up to 17 (three for each of the five entries, and
+// rotations where the line runs in LDS): 5 elements of 8 bytes more per point.
 static constexpr size_t kDenseExtra = 64 * 1024;
+static_assert(5 * 8 * 2 * kDenseMax <= kDenseExtra, "two of the longest lines");
 static __device__ __align__(256) unsigned char scratch[OPO_NOALLOC_SCRATCH_BYTES + kDenseExtra];
 
 static std::mutex g_noalloc_mu;              // one no-allocation call at a time per process

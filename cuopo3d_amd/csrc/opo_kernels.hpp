@@ -123,17 +123,15 @@ int tune_tile_px(bool fp64, int nt, int v);   // pixels per tile of a t-pass var
 // not fit a narrow one.
 int time_variant_for(bool fp64, int nt, int nx, long long pixels);
 int tune_block(bool fp64, int axis, int n, int v);
-int tune_per_cu(bool fp64, int axis, int n, int v);
+int tune_per_cu(bool fp64, int axis, int n, int v);   // persistent workgroups per CU, 0: one unit each
 // Grid of a persistent launch: per_cu workgroups per CU of the current
 // device, at most one per unit.
-unsigned persistent_grid(int units, int per_cu);  // persistent workgroups per CU, 0: one unit each
+unsigned persistent_grid(int units, int per_cu);
 
 // Consecutive t-planes of one field that one workgroup of xy variant v
-// transforms.  Lines of at most 32 points are single register DFTs, one
-// task per line, so one 32 x 32 plane gives a 256-thread workgroup 32
-// tasks per phase; variants 3-5 of NX <= 32 take 256 / NX planes (256
-// tasks), the others one plane.  Every supported NT (16 and up) is a
-// multiple of the group.
+// transforms.  A plane of 16 or 32 points has one or two waves of lines, so
+// variants 3-5 of NX <= 32 take 256 / NX planes, the others one.  Every supported
+// NT (16 and up) is a multiple of the group.
 __host__ __device__ constexpr int xy_group(int nx, int v) {
     return (nx > 1 && nx <= 32 && v >= 3 && v < 6) ? 256 / nx : 1;
 }
@@ -152,8 +150,8 @@ template <typename T> struct SolveDesc {
     cplx<T> *f[3];
     const cplx<T> *twx, *twt;      // rotation tables (TwShear)
     const cplx<T> *tabT, *tabG;    // D tables (3 x 2nt, stride 2nt), GDD table
-    const cplx<T> *qx, *qy;        // Q factor tables (3 fields, stride 2nx / 2ny)
-    const cplx<T> *qfsx, *qfsy;    // free-space factor tables (s, i)
+    const cplx<T> *qx, *qy;        // Q factor tables (3 fields, stride xy_table_elems)
+    const cplx<T> *qfsx, *qfsy;    // free-space factor tables (s, i), likewise
     int nx, ny, nt, gdd_on, n_slices;
     const cplx<T> *eom;            // modulator table (hi/lo pairs), nullptr when off
     T kc1[3], kc3[3], kh6[3];      // nonlinear step weights (see Rk4Args)

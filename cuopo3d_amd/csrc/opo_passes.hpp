@@ -60,11 +60,12 @@ template <typename T, int NT> constexpr int phase_tasks() {
     else return NT / (Split<NT>::N1 > Split<NT>::N2 ? Split<NT>::N1 : Split<NT>::N2);
 }
 
-// Points of the outer register DFT of a time line, and the threads of a tile
-// that each hold that many samples of one pixel.
+// Points of the outer register DFT of a three-level time line (two-level lines
+// have no register form: 1), and the threads of a tile that each hold that many
+// samples of one pixel.
 template <typename T, int NT> constexpr int outer_radix() {
     if constexpr (three_level<T, NT>()) return Split3<NT>::N1;
-    else return Split<NT>::N1;
+    else return 1;
 }
 template <typename T, int NT, int TX> constexpr int reg_threads() { return TX * NT / outer_radix<T, NT>(); }
 // Waves per SIMD the register form is compiled for.
@@ -92,15 +93,10 @@ template <typename T, int NT, int TX> constexpr int time_stage_elems() {
 // wave-private LDS, 15-40 % slower; 1024 threads per tile; persistent workgroups on 512- to
 // 2048-sample lines, 23-90 % slower, their prefetch registers spilling
 // beside 32- and 64-point register DFTs, also with only the twiddles
-// staged so that 4-pixel tiles fit; for 2048-sample lines, 4- and 8-pixel
-// tiles with one field in LDS at a time and the other two held in
-// registers, 28-240 % slower, the held fields spilling beside the
-// three-level line operator; a fused form whose threads load their
-// outer-level samples of all three fields straight from HBM into
-// registers, take the pointwise step and the outer register DFT before the
-// first LDS write and store straight from the inverse outer DFT (two LDS
-// round trips and two barriers fewer, bitwise the same results): ~245
-// VGPRs, 7-20 % slower on 128- to 2048-sample lines.)
+// staged so that 4-pixel tiles fit; the register form of 64- to 256-sample lines,
+// at most equal and on 32 x 32 x 128 21 against 14.5 us per slice, of 2-pixel
+// 2048-sample tiles, 1650 against 1290, and of 4096 samples, spilling 292 bytes,
+// 1575 against 886.)
 constexpr int kTimeClassic = 9;
 constexpr int kTimeVariants = kTimeClassic + 18;
 template <typename T, int NT, int V> struct TimeVariant {
@@ -454,10 +450,15 @@ __device__ __forceinline__ void nl_plane_slices(const TLine3Args<T> &a, int slic
 // A thread holds the N1 samples of its pixel and sub-index m (t = M n1 + m)
 // of all three fields: it loads them, takes the pointwise step and the outer
 // register DFTs, and only the inner phases go through LDS, one field after
-// the other.  The LDS of one field instead of three lets three workgroups
-// share a CU (NT = 2048: 54 KiB), so that one's HBM traffic runs behind the
-// arithmetic of the others; the classic tile fills a CU's LDS and its phases
-// follow each other.  The same operations per element as the classic tile.
+// the other.  The classic tile fills a CU's LDS with three fields of a narrow
+// tile, and its phases follow each other.  With one field in LDS a 2048-sample
+// tile has four pixels (32-byte runs in HBM) instead of two: 72 KiB and 17 of
+// rotations, 96 VGPRs of field, one workgroup of 8 waves per CU; of the shorter
+// lines several workgroups share a CU, so that one's HBM traffic runs behind the
+// arithmetic of the others (1024 samples: three of four pixels, one of eight;
+// 512 samples: three of four pixels, two of eight).  us per slice, both passes:
+// 128 x 128 x 2048 1290 -> 1130, 64 x 64 x 1024 109 -> 99, 64 x 64 x 512 49.8 -> 47.6.
+// The same operations per element as the classic tile.
 // Rotations staged in LDS where that costs no workgroup of the CU.
 template <typename T, int NT, int TX> constexpr bool reg_stage() {
     constexpr int wgs = reg_waves<T, NT, TX>() * 256 / reg_threads<T, NT, TX>();
@@ -466,6 +467,7 @@ template <typename T, int NT, int TX> constexpr bool reg_stage() {
 template <typename T, int NT, int TX, bool PHASE>
 __device__ __forceinline__ void nl_time_reg(const TLine3Args<T> &a, int nx, int ny, int tile,
                                             const cplx<T> *__restrict__ tw, cplx<T> *lds, cplx<T> *twl, int stop) {
+    static_assert(three_level<T, NT>(), "the outer radix is that of the three-level split");
     using L = TimeTile<T, NT, TX>;
     constexpr int N1 = outer_radix<T, NT>(), M = NT / N1, BS = reg_threads<T, NT, TX>();
     constexpr bool STW = reg_stage<T, NT, TX>();
@@ -502,10 +504,7 @@ __device__ __forceinline__ void nl_time_reg(const TLine3Args<T> &a, int nx, int 
             for (int k = 0; k < N1; ++k) lds[L::at((M * k + m) * TX) + l] = v[f][k];
             __syncthreads();
             const LineSet<T> ls{lds, 0, a.tab0 + (f - a.first_field) * a.tab_stride, 0, 1};
-            if constexpr (three_level<T, NT>())
-                line_inner3<T, NT, 1, TX, L::PAD, L::G, +1, true, TwShear>(ls, TX, rot, tid, BS);
-            else
-                line_inner2<T, NT, 1, TX, L::PAD, +1, false, true>(ls, TX, tid, BS);
+            line_inner3<T, NT, 1, TX, L::PAD, L::G, +1, true, TwShear>(ls, TX, rot, tid, BS);
             // a thread reads back, and for the next field overwrites, only
             // the slots that it wrote
 #pragma unroll

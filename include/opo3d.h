@@ -246,7 +246,7 @@ int opo_profile_trips(opo_solve *s, int n, double ms[OPO_N_STAGES],
  * shapes are compile-time constants, DtypesConsts.cuh:45-48).  For the
  * solve's grid and precision, times every compiled variant of the fused
  * t pass (tile width x block size, one tile per workgroup or persistent
- * workgroups) and of the xy pass (block size, persistent workgroups or
+ * workgroups) and of the xy pass (one plane per workgroup or
  * groups of small planes) on stretches of up to 16 slices of the real
  * schedule, the fastest of `reps` stretches counting, by coordinate
  * descent (t, xy, t), and keeps the fastest for all later
