@@ -251,7 +251,7 @@ template <typename T> struct SolveT final : SolveImpl {
                 dense_fill<T>(n, -1, *w8, increment, [&](int i, T re, T im, unsigned l) {
                     h[o_ + i] = C{re, im};
                     if (sizeof(T) == 4) lo[i] = l;
-                }, (double)dense_c<T>(n / 8));
+                }, (double)dense_c<T>(n / 8), true);
                 return;
             }
             const double att = std::exp(la);

@@ -25,7 +25,7 @@ template <int N> void table(const char *label, double phase, double la) {
     std::vector<cl> M(2 * N), r(N), x(N), v(N), o(N), want(N);
     dense_fill<double>(N, -1, w, [&](int k, dense_acc<double> &re, dense_acc<double> &im) {
         dense_increment<dense_acc<double>>(ph[k], std::expm1((dense_acc<double>)-la), re, im);
-    }, [&](int i, double re, double im, unsigned) { M[i] = cl(re, im); }, dense_c<double>(N1));
+    }, [&](int i, double re, double im, unsigned) { M[i] = cl(re, im); }, dense_c<double>(N1), true);
     for (int k1 = 0; k1 < N1; ++k1) M[16 * k1 + 7] += (LD)dense_c<double>(N1);
     for (int j = 0; j < N; ++j) r[j] = std::polar((LD)1, 2 * pi * j / N);
     std::mt19937_64 rng(N);
