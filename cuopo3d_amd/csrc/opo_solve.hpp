@@ -236,13 +236,18 @@ template <typename T> struct SolveT final : SolveImpl {
             if (ny != nx) ry.fill(ny);
             wy = ny == nx ? &rx : &ry;
         }
-        auto put_xy = [&](size_t o_, const LineShape &s, const DenseRootsOf<A> *w8, double la, auto phase) {
+        DenseHalf<A> half[kDenseMax];   // of the phases of the last dense table
+        auto put_xy = [&](size_t o_, const LineShape &s, const DenseRootsOf<A> *w8, double la, auto phase,
+                          bool same_phase = false) {
             const int n = s.n();
             if (w8) {
                 unsigned *lo = reinterpret_cast<unsigned *>(h + o_ + 2 * (size_t)n);
                 const A am1 = std::expm1((A)la);
                 A er[kDenseMax], ei[kDenseMax];   // the entry times n, minus 1; even in the frequency
-                for (int k = 0; k <= n / 2; ++k) dense_increment<A>(phase(k), am1, er[k], ei[k]);
+                for (int k = 0; k <= n / 2; ++k) {
+                    if (!same_phase) half[k] = dense_half<A>(phase(k));
+                    dense_increment(half[k], am1, er[k], ei[k]);
+                }
                 auto increment = [&](int k, A &re, A &im) {
                     const int m = k <= n / 2 ? k : n - k;
                     re = er[m];
@@ -284,6 +289,9 @@ template <typename T> struct SolveT final : SolveImpl {
         const double dfX = nx > 1 ? 1.0 / (p.dx * nx) : 0.0;
         const double dfY = ny > 1 ? 1.0 / (p.dy * ny) : 0.0;
         const double pi2 = 9.869604401089358618834490999876151;  // pi^2
+        // Square cells on a square plane: the phases of y are those of x, and the
+        // free-space tables, without absorption, are the same.
+        const bool square = nx == ny && dfX == dfY;
         for (int f = 0; f < 3; ++f) {
             const double qk = -p.dz * (2.0 * pi2 / p.kdiff[f]);
             put_xy(o.qx + (size_t)f * xy_table_elems<T>(nx), lx, wx, -0.5 * p.alpha[f] * p.dz, [&](int k) {
@@ -293,7 +301,7 @@ template <typename T> struct SolveT final : SolveImpl {
             put_xy(o.qy + (size_t)f * xy_table_elems<T>(ny), ly, wy, 0.0, [&](int k) {
                 const double fy = signed_freq(k, ny);
                 return qk * (dfY * dfY * fy * fy);
-            });
+            }, square);
         }
         // Free space on s and i: exp(+i L 2 pi^2/k (dfX^2 fx^2 + dfY^2 fy^2)), no
         // absorption (Solver3D.cuh:305-323), normalised by 1/(NX NY) (:102-119).
@@ -303,6 +311,11 @@ template <typename T> struct SolveT final : SolveImpl {
                 const double fx = signed_freq(k, nx);
                 return qk * (dfX * dfX * fx * fx);
             });
+            if (square) {
+                const C *fx = h + o.fx + (size_t)f * xy_table_elems<T>(nx);
+                std::copy(fx, fx + xy_table_elems<T>(nx), h + o.fy + (size_t)f * xy_table_elems<T>(ny));
+                continue;
+            }
             put_xy(o.fy + (size_t)f * xy_table_elems<T>(ny), ly, wy, 0.0, [&](int k) {
                 const double fy = signed_freq(k, ny);
                 return qk * (dfY * dfY * fy * fy);
