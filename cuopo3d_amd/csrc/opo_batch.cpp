@@ -534,11 +534,12 @@ struct opo_batch {
             const int rc = time_key(key.first, key.second, reps, ms, launches);
             if (rc) return rc;
             // per-slice stages: the mean over the trip's launches (solves
-            // with fewer slices drop out of the later launches)
+            // with fewer slices drop out of the later launches; plane-wave
+            // solves have one launch for all slices)
             auto per_slice = [&](bool t_pass) {
                 double sum = 0.0;
                 int nl = 0;
-                for (int k = 0; k < n_slices; ++k) {
+                for (int k = 0; k < (t_pass && key.second < 0 ? 1 : n_slices); ++k) {
                     const double b = class_bytes(3, 2, [&](const BatchEntry *e) {
                         return (t_pass ? tclass(e) == key.second : in_xy(e, key.second)) && e->p.n_slices > k;
                     });
